@@ -30,7 +30,7 @@ int wave_x_apply(const Geom& g, int nbt, cpx<T>* box, const T* vx, const cpx<T>*
   if constexpr (sizeof(T) == 4) {
     // staged tiles where they move in pairs (n2 n3 even) and several bands share a
     // workgroup: 72^3, 133 bands 130 -> 111 us (90^3, 160 bands 310 -> 235)
-    const size_t lds = kXWaves * (size_t)es * 8 + ((size_t)g.n1 + 2 * (size_t)(g.na + 2) * lines) * sizeof(cpx<T>);
+    const size_t lds = stage_lds_bytes(g.n1, g.na, lines, kXWaves * (size_t)es * 8, sizeof(cpx<T>));
     if (bgroup >= 4 && g.n2 * g.n3 % 2 == 0 && lds <= kLdsPerCu / 2) {
 #define GW_CASE(M, S)                                                                                           \
   case (M) * (S):                                                                                               \

@@ -98,6 +98,14 @@ k_xpass_wave(Geom g, int nbt, int bgroup, cpx<T>* __restrict__ box, const T* __r
 
 constexpr int kXTilePad = 0;  // extra elements per row of the staged x-pass tiles (1, 2, 4 measured slower)
 
+// LDS of k_xpass_stage: exchange areas (ex_bytes, a multiple of 16), the n x
+// twiddles, two tiles of na + 2 rows. The twiddles take a whole number of pairs, so
+// that the tiles start on 16 bytes for odd n too: FP32 tiles move as pairs.
+constexpr int stage_tw(int n) { return (n + 1) & ~1; }
+inline size_t stage_lds_bytes(int n, int na, int lines, size_t ex_bytes, size_t elem) {
+  return ex_bytes + (stage_tw(n) + 2 * (size_t)(na + 2) * (lines + kXTilePad)) * elem;
+}
+
 // P2 with the band's sphere planes staged through LDS. A workgroup of NWX waves
 // owns a chunk of LC = NWX*LW yz-lines; one band's na planes of that chunk form
 // a tile of na rows x LC contiguous elements, which arrives with row-contiguous
@@ -117,16 +125,19 @@ k_xpass_stage(Geom g, int nbt, int bgroup, cpx<T>* __restrict__ box, const T* __
   constexpr int NT = 64 * NWX;
   // FP32 tiles move in pairs of adjacent lines (16-byte accesses): every tile row
   // starts at an even line (PAIR: n2*n3 is even, as LC and j0 are), so a pair never
-  // straddles a row or the last line
+  // straddles a row or the last line; in LDS the tiles start on 16 bytes and their
+  // rows are whole pairs
   constexpr int PK = (sizeof(T) == 4 && LC % 2 == 0 && PAIR) ? 2 : 1;
   using SV = typename std::conditional<PK == 2, cpx2f, cpx<T>>::type;
   constexpr int LCU = LC / PK;                  // staging units per tile row
   constexpr int KS = (N * LCU + NT - 1) / NT;   // staged units per thread (na <= N rows)
   constexpr int LDT = LC + kXTilePad;           // tile row stride
+  static_assert(PK == 1 || (LDT % 2 == 0 && (NWX * W::E_PER_WAVE * sizeof(typename W::EX) +
+                                             stage_tw(N) * sizeof(cpx<T>)) % sizeof(SV) == 0), "pairs on 16 bytes");
   extern __shared__ __align__(16) unsigned char smem_raw[];
   typename W::EX* E = reinterpret_cast<typename W::EX*>(smem_raw);
   cpx<T>* tw = reinterpret_cast<cpx<T>*>(E + NWX * W::E_PER_WAVE);  // E_PER_WAVE is even
-  cpx<T>* tiles = tw + N;                        // 2 x (na + 2) rows of LC
+  cpx<T>* tiles = tw + stage_tw(N);              // 2 x (na + 2) rows of LC
   const long wid = xcd_work_id(total);
   if (wid < 0) return;
   const int chunk = (int)(wid % nchunk), bgi = (int)(wid / nchunk);

@@ -1161,9 +1161,8 @@ static int launch_wave_path_n(Plan& P, const Geom& g, int nbt, const cpx<T>* c, 
   const int nchunk = (n23 + lines_per_wg - 1) / lines_per_wg;
   const long xtotal = (long)nchunk * ((nbt + bgroup - 1) / bgroup);
   const dim3 xgrid((unsigned)(8 * ((xtotal + 7) / 8)));
-  const size_t stage_lds =
-      (size_t)nwx * W::E_PER_WAVE * sizeof(typename W::EX) +
-      (N + 2 * (size_t)(P.na + 2) * (lines_per_wg + kXTilePad)) * sizeof(cpx<T>);
+  const size_t stage_lds = stage_lds_bytes(N, P.na, lines_per_wg, (size_t)nwx * W::E_PER_WAVE * sizeof(typename W::EX),
+                                           sizeof(cpx<T>));
   if (xs.mode == 1 && stage_lds <= (size_t)std::min(P.lds_max, kMaxLds)) {
     if (nwx == 8)
       hipLaunchKernelGGL((k_xpass_stage<T, N, C::M, C::S, 8>), xgrid, dim3(512), stage_lds, st, g, nbt, bgroup,
