@@ -42,16 +42,11 @@ HARTREE_EV = 27.211386245988
 BOHR_ANG = 0.529177210903
 HBAR2_2M = HARTREE_EV / 2.0 * BOHR_ANG**2
 
-_WS: dict[tuple, torch.Tensor] = {}
 
-
-def _scratch(device: torch.device, nbytes: int, tag: str) -> torch.Tensor:
-    key = (tag, device.index)
-    ws = _WS.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
-        _WS[key] = ws
-    return ws
+def _scratch(device: torch.device, nbytes: int) -> torch.Tensor:
+    """Workspace of one call. The allocator keeps and reuses its memory per stream, so
+    gradients taken on two streams never write into each other's."""
+    return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
 
 
 def _symmetric(d: torch.Tensor) -> bool:
@@ -111,7 +106,7 @@ def adjoint_v(op: HOperator, c: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
     if info[2] != 2:  # no wave-line path on this box: transform to r and sum
         return _adjoint_v_real_space(op, c, g, gv)
     need = int(L.lib().gw_hpsi_adjoint_v_workspace_bytes(plan.handle, nb, prec))
-    ws = _scratch(c.device, need, "adjv")
+    ws = _scratch(c.device, need)
     L.check(L.lib().gw_hpsi_adjoint_v(plan.handle, prec, c.data_ptr(), c.stride(1), c.stride(0),
                                       g.data_ptr(), g.stride(1), g.stride(0), nb, gv.data_ptr(),
                                       ws.data_ptr(), ws.numel(), L.stream_ptr(c.device)),
@@ -235,7 +230,7 @@ class _ProjPhaseFn(torch.autograd.Function):
         gp = grad_p.to(torch.complex128).contiguous()
         gtau = torch.zeros(ctx.na, 3, dtype=torch.float64, device=p.device)
         need = int(L.lib().gw_proj_phase_grad_workspace_bytes(nk, nproj))
-        ws = _scratch(p.device, need, "phase")
+        ws = _scratch(p.device, need)
         L.check(L.lib().gw_proj_phase_grad(nk, nproj, npw_max, ctx.na, gp.data_ptr(), p.data_ptr(),
                                            kpg.data_ptr(), atom_index.data_ptr(), gtau.data_ptr(),
                                            ws.data_ptr(), ws.numel(), L.stream_ptr(p.device)),
@@ -291,7 +286,7 @@ class _VlocGFn(torch.autograd.Function):
         gv = grad_vg.to(torch.complex128).contiguous()
         gtau = torch.zeros(na, 3, dtype=torch.float64, device=pos.device)
         need = int(L.lib().gw_vloc_g_grad_workspace_bytes(na))
-        ws = _scratch(pos.device, need, "vloc")
+        ws = _scratch(pos.device, need)
         L.check(L.lib().gw_vloc_g_grad(na, npts, pos.data_ptr(), sidx.data_ptr(), tables.data_ptr(),
                                        g_cart.data_ptr(), ctx.volume, gv.data_ptr(), gtau.data_ptr(),
                                        ws.data_ptr(), ws.numel(), L.stream_ptr(pos.device)),

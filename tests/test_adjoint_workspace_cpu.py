@@ -1,0 +1,73 @@
+"""Workspaces of the adjoint and eigensolver entry points, with a stand-in for the
+library that records the pointers it is given: calls that overlap (two streams) get
+memory of their own, and one call's memory is bounded."""
+
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from gradwave_amd import _lib as L
+from gradwave_amd import adjoint as A
+
+
+class _Library:
+    """gw_hpsi_adjoint_v and gw_proj_phase_grad, recording (workspace, bytes); ``during``
+    runs inside the first call, as another stream's call would."""
+
+    def __init__(self, bytes_of, during=None):
+        self.bytes_of, self.during, self.calls = bytes_of, during, []
+
+    def gw_plan_info(self, handle, prec, info, n):
+        info[2] = 2
+        return 0
+
+    def gw_hpsi_adjoint_v_workspace_bytes(self, handle, nb, prec):
+        return self.bytes_of(nb)
+
+    def gw_proj_phase_grad_workspace_bytes(self, nk, nproj):
+        return self.bytes_of(nproj)
+
+    def _call(self, **kw):
+        self.calls.append(SimpleNamespace(**kw))
+        if self.during is not None and len(self.calls) == 1:
+            self.during()
+        return 0
+
+    def gw_hpsi_adjoint_v(self, handle, prec, c, ldc, sc, g, ldg, sg, nb, gv, ws, nbytes, stream):
+        return self._call(c=c, g=g, nb=nb, ws=ws, bytes=nbytes)
+
+    def gw_proj_phase_grad(self, nk, nproj, npw, na, gp, p, kpg, ai, gtau, ws, nbytes, stream):
+        return self._call(ws=ws, bytes=nbytes)
+
+
+@pytest.fixture
+def install(monkeypatch):
+    def put(lib):
+        monkeypatch.setattr(L, "lib", lambda: lib)
+        monkeypatch.setattr(L, "stream_ptr", lambda device=None: 0)
+        return lib
+    return put
+
+
+def _block(nb):
+    return torch.zeros(2, nb, 7, dtype=torch.complex128)
+
+
+def _disjoint(a, b):
+    return a.ws + a.bytes <= b.ws or b.ws + b.bytes <= a.ws
+
+
+def test_overlapping_v_adjoints_do_not_share_a_workspace(install):
+    op = SimpleNamespace(fwd=SimpleNamespace(plan=SimpleNamespace(handle=None)), shape=(4, 4, 4))
+    lib = install(_Library(lambda nb: 4096 * nb, lambda: A.adjoint_v(op, _block(2), _block(2))))
+    A.adjoint_v(op, _block(3), _block(3))
+    assert len(lib.calls) == 2 and _disjoint(*lib.calls)
+
+
+def test_overlapping_phase_adjoints_do_not_share_a_workspace(install):
+    p = torch.zeros(2, 3, 7, dtype=torch.complex128)
+    ctx = SimpleNamespace(saved_tensors=(p, torch.zeros(2, 7, 3), torch.zeros(3, dtype=torch.int64)), na=1)
+    lib = install(_Library(lambda n: 4096 * n, lambda: A._ProjPhaseFn.backward(ctx, p)))
+    A._ProjPhaseFn.backward(ctx, p)
+    assert len(lib.calls) == 2 and _disjoint(*lib.calls)

@@ -1,0 +1,36 @@
+"""The V(r) adjoint of two operators on two streams at once, against the same calls in turn."""
+
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from gpu_cases import dev, rand_block, say
+from test_gpu_box_lengths import _gpu_h, _si2
+
+pytestmark = pytest.mark.gpu
+
+from gradwave_amd import adjoint as A  # noqa: E402
+
+
+def _problem(shape, nb, seed):
+    s = _si2(shape)
+    cpu, _, h = _gpu_h(s, toeplitz="off")
+    c, g = (rand_block(cpu.nk, nb, cpu.npw_max, cpu.mask, seed=seed + i).to(dev()) for i in range(2))
+    return SimpleNamespace(fwd=h, shape=s.shape), c, g
+
+
+def test_v_adjoints_on_two_streams():
+    say("V adjoint on two streams")
+    problems = [_problem((30, 28, 27), 40, 90), _problem((36, 36, 36), 33, 92)]
+    want = [A.adjoint_v(*p) for p in problems]
+    streams = [torch.cuda.Stream() for _ in problems]
+    torch.cuda.synchronize()
+    got = [[], []]
+    for _ in range(6):
+        for i, (p, st) in enumerate(zip(problems, streams)):
+            with torch.cuda.stream(st):
+                got[i].append(A.adjoint_v(*p))
+    torch.cuda.synchronize()
+    for i, w in enumerate(want):
+        assert all(torch.equal(x, w) for x in got[i])
