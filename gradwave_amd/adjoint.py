@@ -91,7 +91,10 @@ def _adjoint_v_real_space(op: HOperator, c: torch.Tensor, g: torch.Tensor, gv: t
 
 
 def adjoint_v(op: HOperator, c: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
-    """(1/N) sum_{k,b} Re[conj(N ifftn g) (N ifftn c)] on the natural box, float64."""
+    """(1/N) sum_{k,b} Re[conj(N ifftn g) (N ifftn c)] on the natural box, float64, in
+    band chunks of at most GW_LIB_FFT_BUDGET bytes of workspace."""
+    from gradwave_amd.hamiltonian import _LIB_FFT_BUDGET_BYTES
+
     plan = op.fwd.plan
     prec = L.precision_of(c.dtype)
     c = c if c.stride(2) == 1 else c.contiguous()
@@ -105,12 +108,22 @@ def adjoint_v(op: HOperator, c: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
     L.check(L.lib().gw_plan_info(plan.handle, prec, info, 3), "gw_plan_info")
     if info[2] != 2:  # no wave-line path on this box: transform to r and sum
         return _adjoint_v_real_space(op, c, g, gv)
-    need = int(L.lib().gw_hpsi_adjoint_v_workspace_bytes(plan.handle, nb, prec))
-    ws = _scratch(c.device, need)
-    L.check(L.lib().gw_hpsi_adjoint_v(plan.handle, prec, c.data_ptr(), c.stride(1), c.stride(0),
-                                      g.data_ptr(), g.stride(1), g.stride(0), nb, gv.data_ptr(),
+    lib = L.lib()
+
+    def need(n: int) -> int:
+        return int(lib.gw_hpsi_adjoint_v_workspace_bytes(plan.handle, n, prec))
+
+    # both boxes of the block at once, or of as many bands as the budget holds
+    step = max(1, min(nb, nb * _LIB_FFT_BUDGET_BYTES // need(nb)))
+    while step > 1 and need(step) > _LIB_FFT_BUDGET_BYTES:
+        step -= 1
+    ws = _scratch(c.device, need(step))
+    for b0 in range(0, nb, step):
+        cb, gb = c[:, b0:b0 + step], g[:, b0:b0 + step]
+        L.check(lib.gw_hpsi_adjoint_v(plan.handle, prec, cb.data_ptr(), cb.stride(1), cb.stride(0),
+                                      gb.data_ptr(), gb.stride(1), gb.stride(0), int(cb.shape[1]), gv.data_ptr(),
                                       ws.data_ptr(), ws.numel(), L.stream_ptr(c.device)),
-            "gw_hpsi_adjoint_v")
+                "gw_hpsi_adjoint_v")
     return gv
 
 

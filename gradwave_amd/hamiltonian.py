@@ -31,8 +31,8 @@ _TOEPLITZ_ON_GPU = os.environ.get("GW_TOEPLITZ_ON_GPU", "0") == "1"
 _TOEPLITZ_M_BUDGET_BYTES = int(os.environ.get("GW_TOEPLITZ_BUDGET", str(4 << 30)))
 _TOEP_TRIAL_MARGIN = 0.7
 _TOEP_TRIAL: dict[tuple, bool] = {}
-# Device bytes one band chunk of the library-FFT local term may hold (box,
-# psi(r) and the transformed box).
+# Device bytes one band chunk of the library-FFT local term (box, psi(r) and the
+# transformed box) or of the V(r) adjoint (both boxes and the partial sums) may hold.
 _LIB_FFT_BUDGET_BYTES = int(os.environ.get("GW_LIB_FFT_BUDGET", str(2 << 30)))
 
 

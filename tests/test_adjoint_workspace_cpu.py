@@ -71,3 +71,21 @@ def test_overlapping_phase_adjoints_do_not_share_a_workspace(install):
     lib = install(_Library(lambda n: 4096 * n, lambda: A._ProjPhaseFn.backward(ctx, p)))
     A._ProjPhaseFn.backward(ctx, p)
     assert len(lib.calls) == 2 and _disjoint(*lib.calls)
+
+
+def test_v_adjoint_goes_in_band_chunks_under_the_budget(install, monkeypatch):
+    from gradwave_amd import hamiltonian
+
+    monkeypatch.setattr(hamiltonian, "_LIB_FFT_BUDGET_BYTES", 3500)
+    op = SimpleNamespace(fwd=SimpleNamespace(plan=SimpleNamespace(handle=None)), shape=(4, 4, 4))
+    # one band is above the budget, three bands fit, a partial per group of two bands
+    for per_band, group, chunks in ((9000, 0, [1] * 8), (1000, 0, [3, 3, 2]), (1000, 600, [2, 2, 2, 2]), (10, 0, [8])):
+        lib = install(_Library(lambda nb: per_band * nb + group * ((nb + 1) // 2)))
+        c, g = _block(8), _block(8)
+        A.adjoint_v(op, c, g)
+        assert [x.nb for x in lib.calls] == chunks
+        done = 0
+        for x in lib.calls:
+            assert x.c == c.data_ptr() + done * c.stride(1) * 16 and x.g == g.data_ptr() + done * g.stride(1) * 16
+            assert x.bytes >= lib.bytes_of(x.nb) and x.bytes <= max(3500, lib.bytes_of(1))
+            done += x.nb

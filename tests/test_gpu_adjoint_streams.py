@@ -34,3 +34,18 @@ def test_v_adjoints_on_two_streams():
     torch.cuda.synchronize()
     for i, w in enumerate(want):
         assert all(torch.equal(x, w) for x in got[i])
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.complex128, 1e-12), (torch.complex64, 1e-12)])
+def test_v_adjoint_in_band_chunks(dtype, tol, monkeypatch):
+    """Chunks sum in another order only (FP64 sums of the same products)."""
+    from gradwave_amd import hamiltonian
+
+    say(f"V adjoint in chunks {dtype}")
+    op, c, g = _problem((30, 28, 27), 19, 94)
+    c, g = c.to(dtype), g.to(dtype)
+    whole = A.adjoint_v(op, c, g)
+    calls = 2 * c.shape[0] * 19 * 30 * 28 * 27 * c.element_size()  # above the whole block's two boxes
+    monkeypatch.setattr(hamiltonian, "_LIB_FFT_BUDGET_BYTES", calls // 7)
+    parts = A.adjoint_v(op, c, g)
+    assert float((parts - whole).abs().max() / whole.abs().max()) < tol
