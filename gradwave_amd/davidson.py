@@ -130,8 +130,9 @@ def _cholinv_torch(g: torch.Tensor):
 def _cholinv(g: torch.Tensor):
     """(L^-1, info) of the (nk, n, n) Gram matrices: all k in one launch up to
     ``chol_max_n`` on the GPU (36 k, n = 24: torch's potrf, solve and copies take
-    seven launches; a Si8 36 k-point solve 133 -> 114 ms), torch elsewhere."""
-    if g.is_cuda and g.shape[-1] <= LA.chol_max_n():
+    seven launches; a Si8 36 k-point solve 133 -> 114 ms), torch elsewhere, for an
+    empty block too."""
+    if g.is_cuda and 0 < g.shape[-1] <= LA.chol_max_n():
         return LA.cholesky_inverse([g])[0]
     return _cholinv_torch(g)
 

@@ -190,3 +190,12 @@ def test_cholesky_inverse_request_on_both_sides_of_the_kernel(nk, n):
     li = linv.cpu()
     assert float((li @ g @ li.mH - eye).abs().max()) < 1e-12
     assert float(li.triu(1).abs().max()) == 0.0
+
+
+def test_orthonormalisation_of_an_empty_block():
+    """No rows: no Cholesky job, an empty result and clear flags, as with torch."""
+    from gradwave_amd.davidson import _cholqr2_dev
+
+    say("cholqr2 of no rows")
+    q, flags = _cholqr2_dev(torch.zeros(2, 0, 50, dtype=torch.complex128, device=dev()))
+    assert tuple(q.shape) == (2, 0, 50) and int(flags.abs().max()) == 0
