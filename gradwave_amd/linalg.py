@@ -163,9 +163,6 @@ def rcombine(u: torch.Tensor, y: torch.Tensor, out: torch.Tensor | None = None, 
     return out
 
 
-_HEEV_WS: dict[tuple, torch.Tensor] = {}
-
-
 def heev_max_n() -> int:
     return int(L.lib().gw_heev_max_n())
 
@@ -199,11 +196,7 @@ def eigh_lowest(mats: list, nevs: list) -> list:
         out.append((w, u))
         jobs.append((s, w, u, nk, m, nev, need))
     total = sum(j[3] * j[6] for j in jobs)
-    key = (dev.type, dev.index)
-    ws = _HEEV_WS.get(key)
-    if ws is None or ws.numel() < total:
-        ws = torch.empty(max(total, 1 << 20), dtype=torch.uint8, device=dev)
-        _HEEV_WS[key] = ws
+    ws = torch.empty(total, dtype=torch.uint8, device=dev)  # of the call: two streams never share it
     count = sum(j[3] for j in jobs)
     arr = (L.HeevJob * count)()
     off, i = ws.data_ptr(), 0

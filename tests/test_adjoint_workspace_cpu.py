@@ -89,3 +89,29 @@ def test_v_adjoint_goes_in_band_chunks_under_the_budget(install, monkeypatch):
             assert x.c == c.data_ptr() + done * c.stride(1) * 16 and x.g == g.data_ptr() + done * g.stride(1) * 16
             assert x.bytes >= lib.bytes_of(x.nb) and x.bytes <= max(3500, lib.bytes_of(1))
             done += x.nb
+
+
+def test_overlapping_eigensolves_do_not_share_a_workspace(monkeypatch):
+    from gradwave_amd import linalg as LA
+
+    jobs = []
+
+    class Lib:
+        def gw_heev_workspace_bytes(self, n, nev):
+            return 4096 * n
+
+        def gw_heev_max_n(self):
+            return 512
+
+        def gw_heev_batched(self, count, arr, stream):
+            jobs.append([(arr[i].ws, 4096 * arr[i].n) for i in range(count)])
+            if len(jobs) == 1:  # another stream's call
+                LA.eigh_lowest([torch.zeros(2, 3, 3, dtype=torch.complex128)], [1])
+            return 0
+
+    monkeypatch.setattr(L, "lib", lambda: Lib())
+    monkeypatch.setattr(L, "stream_ptr", lambda device=None: 0)
+    monkeypatch.setattr(L, "require_gpu", lambda t, name: None)
+    LA.eigh_lowest([torch.zeros(3, 5, 5, dtype=torch.complex128)], [2])
+    spans = sorted(jobs[0] + jobs[1])
+    assert len(spans) == 5 and all(a[0] + a[1] <= b[0] for a, b in zip(spans, spans[1:]))
