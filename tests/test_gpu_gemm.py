@@ -254,3 +254,59 @@ def test_empty_contraction_is_zero(dtype):
     v = torch.zeros(2, 0, 5, dtype=dtype, device=dev())
     r = LA.combine(u, v, out=z, beta=0.5)
     assert float((r - 1.0).abs().max().cpu()) == 0.0
+
+
+def _component_bound(terms, dtype):
+    """Rounding of a sum of real products a component at a time: (number of products)
+    u sum |products|, once for the kernel and once for the float64 reference."""
+    u = 2.0 ** -53 if dtype == torch.complex128 else 2.0 ** -24
+    n = sum(a.shape[-1] for a, _ in terms)
+    return (n + 4) * (u + 2.0 ** -53) * sum(torch.matmul(a.abs(), b.abs().mT.contiguous()) for a, b in terms)
+
+
+@pytest.mark.parametrize("dtype", [torch.complex128, torch.complex64])
+def test_default_tiles_keep_small_components(dtype):
+    """Vectors whose imaginary part is 1e-8 of the real one: each component of the
+    default contractions carries its own rounding only, at every tile of the rule
+    (rows of 16, 32 and 64 or 96) and short and long sums."""
+    say(f"gemm default tiles by component {dtype}")
+
+    def narrow(nk, rows, cols, seed):
+        z = _rand(nk, rows, cols, seed=seed, dtype=torch.complex128)
+        return torch.complex(z.real, 1e-8 * z.imag).to(dtype)
+
+    def parts(z):
+        return z.real.double(), z.imag.double()
+
+    for (M, N, K) in [(8, 5, 70), (33, 40, 4097), (160, 160, 20001), (320, 192, 2500), (864, 480, 4097)]:
+        x, y = narrow(1, M, K, 1), narrow(1, N, K, 2)
+        got = LA.inner(x.to(dev()), y.to(dev())).cpu()
+        (xr, xi), (yr, yi) = parts(x), parts(y)
+        for have, terms in ((got.real, ((xr, yr), (xi, yi))), (got.imag, ((xr, yi), (-xi, yr)))):
+            want = sum(torch.matmul(a, b.mT.contiguous()) for a, b in terms)
+            assert bool(((have.double() - want).abs() <= _component_bound(terms, dtype)).all()), (M, N, K)
+    for (A, G, J) in [(7, 65, 100), (33, 129, 96), (160, 500, 300), (288, 300, 96), (480, 640, 1000)]:
+        u, y = narrow(1, J, A, 3), narrow(1, J, G, 4)
+        for conj_u in (False, True):
+            got = LA.combine(u.to(dev()), y.to(dev()), conj_u=conj_u).cpu()
+            (ur, ui), (yr, yi) = (tuple(p.mT.contiguous() for p in parts(z)) for z in (u, y))
+            ui = -ui if conj_u else ui
+            for have, terms in ((got.real, ((ur, yr), (-ui, yi))), (got.imag, ((ur, yi), (ui, yr)))):
+                want = sum(torch.matmul(a, b.mT.contiguous()) for a, b in terms)
+                assert bool(((have.double() - want).abs() <= _component_bound(terms, dtype)).all()), (A, G, J, conj_u)
+
+
+def test_default_tiles_do_not_overflow_early():
+    """FP32 operands whose two components each fit, and their sum does not."""
+    say("gemm default tiles near the FP32 range")
+    for (M, N, K) in [(33, 40, 20001), (320, 192, 2500)]:
+        for sign in (1, -1):  # conj(x) y is 4e8 in one component, 0 in the other
+            x = torch.full((1, M, K), 2e38 * (1 + sign * 1j), dtype=torch.complex64)
+            y = torch.full((1, N, K), 1e-30 * (1 + 1j), dtype=torch.complex64)
+            got = LA.inner(x.to(dev()), y.to(dev())).cpu()
+            z = LA.combine(x.mT.contiguous()[:, :300].to(dev()), y.mT.contiguous()[:, :300].to(dev()),
+                           conj_u=True).cpu()
+            for have, n in ((got, K), (z, 300)):
+                assert bool(torch.isfinite(torch.view_as_real(have)).all()), (M, N, K)
+                big = have.real if sign > 0 else have.imag
+                assert float((big.double() / (n * 4e8) - 1).abs().max()) < 2 * n * 2.0 ** -24
