@@ -294,17 +294,19 @@ def tune_gemm(workloads, nb: int = 32, reps: int = 5, allow_library: bool = True
 
 # x-pass shapes: mode * 10000 + waves * 100 + bands (mode 1: planes staged through LDS)
 XPASS_SHAPES = (408, 416, 208, 10408, 10416, 10432, 10208)
-WAVE_LENGTHS = (24, 36, 90, 120)  # cubes whose launch shapes are timed; the rule picks for 24 and 36
+XPASS_LENGTHS = (90, 120)  # the cubes whose x pass takes GW_TUNE_XPASS
+WAVE_LENGTHS = (24, 36, 90, 120)  # cubes whose bands per plane item are timed
 
 
 def tune_xpass(workloads, nb: int = 32, reps: int = 5) -> dict:
-    """For each precision, time the local term of the ``workloads`` whose box is a
-    wave-line cube under each x-pass shape and keep the fastest. Returns
-    {"fp64": shape, "fp32": shape} (the current shapes if no workload qualifies)."""
+    """For each precision, time the local term of the ``workloads`` whose box is a 90
+    or 120 cube under each x-pass shape and keep the fastest. Returns
+    {"fp64": shape, "fp32": shape} (the current shapes if no workload qualifies: on
+    other boxes every shape runs the same kernel)."""
     from gradwave_amd.hamiltonian import BatchedHamiltonian
 
     lib = L.lib()
-    users = [w for w in workloads if len(set(w.shape)) == 1 and w.shape[0] in WAVE_LENGTHS]
+    users = [w for w in workloads if len(set(w.shape)) == 1 and w.shape[0] in XPASS_LENGTHS]
     chosen = {"fp64": lib.gw_tune_get(L.GW_TUNE_XPASS, L.GW_FP64),
               "fp32": lib.gw_tune_get(L.GW_TUNE_XPASS, L.GW_FP32)}
     if not users:
