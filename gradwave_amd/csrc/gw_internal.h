@@ -91,7 +91,7 @@ struct Plan {
   int* d_colptr;  // (nproj+1)
   int* d_row;     // nnz
   double* d_val;  // nnz
-  int d_nnz;
+  int d_nnz, d_width;  // entries, and the most in one column
   int flags;     // GW_PLAN_* bits
   int lds_max;   // dynamic LDS bytes available per workgroup
 };
@@ -198,6 +198,7 @@ struct InnerDmul {
   const int* colptr;
   const int* row;
   const double* val;
+  int width;  // most nonzeros in a column of D
   void* u;
   bool done;
 };

@@ -1781,6 +1781,8 @@ extern "C" int gw_plan_set_projectors(gw_plan* h, int nproj, const void* p, cons
     colptr[q + 1] = (int)row.size();
   }
   P.d_nnz = (int)row.size();
+  P.d_width = 0;
+  for (int q = 0; q < nproj; ++q) P.d_width = std::max(P.d_width, colptr[q + 1] - colptr[q]);
   GW_CHECK_HIP(hipMalloc(&P.d_colptr, colptr.size() * sizeof(int)));
   GW_CHECK_HIP(hipMalloc(&P.d_row, std::max<size_t>(1, row.size()) * sizeof(int)));
   GW_CHECK_HIP(hipMalloc(&P.d_val, std::max<size_t>(1, val.size()) * sizeof(double)));
@@ -1994,18 +1996,18 @@ static int apply_t(gw_plan* h, int terms, const cpx<T>* c, long ldc, long sc, cp
     cpx<T>* u = (cpx<T>*)(ws + L.u_off);
     const long pstride = (long)P.nproj * P.npw_max;
     ev = tm.begin();
-    InnerDmul dm{P.d_colptr, P.d_row, P.d_val, u, false};
+    InnerDmul dm{P.d_colptr, P.d_row, P.d_val, P.d_width, u, false};
     int rc = gemm_inner<T>(P.nk, P.nproj, nb, P.npw_max, pr, P.npw_max, pstride, c, ldc, sc, becp, nb,
                            (long)P.nproj * nb, ws + L.part_off, L.part_bytes, st, &dm);
     if (rc) return rc;
     tm.end(ST_BECP, ev);
-    ev = tm.begin();
     if (!dm.done) {
+      ev = tm.begin();
       hipLaunchKernelGGL(k_dmul<T>, dim3(grid_blocks((long)P.nproj * nb, 256), P.nk), dim3(256), 0, st, P.nproj,
                          nb, P.d_colptr, P.d_row, P.d_val, becp, u);
       GW_CHECK_HIP(hipGetLastError());
+      tm.end(ST_DMUL, ev);
     }
-    tm.end(ST_DMUL, ev);
     ev = tm.begin();
     rc = gemm_combine<T>(P.nk, nb, P.npw_max, P.nproj, u, nb, (long)P.nproj * nb, 0, pr, P.npw_max, pstride,
                          out, ldo, so, base ? T(1) : T(0), st);
@@ -2653,7 +2655,7 @@ static int batch_apply_t(gw_batch* b, const BatchBind& s, hipStream_t st) {
     cpx<T>* becp = (cpx<T>*)(B.ws + L.becp_off);
     cpx<T>* u = (cpx<T>*)(B.ws + L.u_off);
     const long pstride = (long)P.nproj * P.npw_max;
-    InnerDmul dm{P.d_colptr, P.d_row, P.d_val, u, false};
+    InnerDmul dm{P.d_colptr, P.d_row, P.d_val, P.d_width, u, false};
     int rc = gemm_inner<T>(P.nk, P.nproj, B.nb, P.npw_max, pr, P.npw_max, pstride, (const cpx<T>*)B.c, B.ldc, B.sc,
                            becp, B.nb, (long)P.nproj * B.nb, B.ws + L.part_off, L.part_bytes, ls, &dm);
     if (rc == GW_OK) {

@@ -73,8 +73,9 @@ int gw_plan_set_flags(gw_plan* plan, int flags);
 /* With GW_PLAN_TIMING set, gw_hpsi_apply records HIP events around each of its
  * stages on the launch stream: 0 x-plane inverse (pack, z, y), 1 x pass
  * (x inverse, V, x forward), 2 x-plane forward (y, z, gather, kinetic),
- * 3 projection <p|c>, 4 D multiply, 5 back-projection. This returns the summed
- * milliseconds and call counts per stage (synchronising on pending events). */
+ * 3 projection <p|c>, 4 D multiply (no call where it joins the reduction of 3),
+ * 5 back-projection. This returns the summed milliseconds and call counts per
+ * stage (synchronising on pending events). */
 int gw_plan_stage_times(gw_plan* plan, double* ms, long* calls, int n, int reset);
 /* info[0..14] = active x-planes, max sticks per k, fused plane path (0/1) for
  * `precision` (2 wave-line, 1 LDS plane tile, 0 split), LDS bytes per
