@@ -103,9 +103,11 @@ def main() -> None:
     x64 = W.start_vectors(wl, seed=0)
     x32 = x64.to(torch.complex64)
     tuned = None
-    if not args.no_autotune:
-        from gradwave_amd import autotune
+    from gradwave_amd import autotune
 
+    if args.no_autotune:
+        autotune.load()  # an earlier run's choices, its GEMM tiles among them
+    else:
         t1 = time.perf_counter()
         tiles, wgs = autotune.tune_gemm([wl], nb=nb)
         plane_bands = autotune.tune_plane_bands([wl], nb=nb)

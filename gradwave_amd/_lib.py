@@ -125,7 +125,7 @@ def lib() -> C.CDLL:
         _lib = h
         from gradwave_amd import autotune  # saved radix / split-K choices, if any
 
-        autotune.load()
+        autotune.load(tiles=False)
     return _lib
 
 

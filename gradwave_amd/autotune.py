@@ -17,7 +17,10 @@ the GEMMs (no reference counterpart: the reference uses torch.fft and BLAS).
   (``GW_TUNE_XPASS``, per precision); ``tune_xpass`` times the local term.
 
 Choices persist as JSON (``GW_TUNE_FILE``, default
-``~/.cache/gradwave_amd/tune.json``) and are loaded with the library.
+``~/.cache/gradwave_amd/tune.json``) and are loaded with the library, but for the
+GEMM tiles: one tile serves every size, where the rule picks by shape (those that win
+on 216 atoms take 8 atoms at 36 k-points from 393 to 484 us), and may have three products. A program
+that wants the saved tiles calls ``load``.
 """
 
 from __future__ import annotations
@@ -124,8 +127,11 @@ def current() -> dict:
                             for name, prec in (("fp64", L.GW_FP64), ("fp32", L.GW_FP32))}}
 
 
-def apply(choices: dict) -> None:
+def apply(choices: dict, tiles: bool = True) -> None:
+    """Set the saved choices; with ``tiles`` false the GEMM tiles stay by shape."""
     lib = L.lib()
+    if not tiles:
+        choices = {k: v for k, v in choices.items() if k not in ("gemm_tile", "gemm_tile_combine")}
     for n, a in choices.get("radix", {}).items():
         L.check(lib.gw_tune_set(L.GW_TUNE_RADIX, int(n), int(a)), "gw_tune_set")
     if "gemm_wgs" in choices:
@@ -148,13 +154,13 @@ def apply(choices: dict) -> None:
             L.check(lib.gw_tune_set(L.GW_TUNE_PLANE_BANDS, prec + 512, int(p3)), "gw_tune_set")
 
 
-def load(path: str | None = None) -> dict | None:
+def load(path: str | None = None, tiles: bool = True) -> dict | None:
     path = path or tune_file()
     if not os.path.exists(path):
         return None
     with open(path) as f:
         choices = json.load(f)
-    apply(choices)
+    apply(choices, tiles)
     return choices
 
 
