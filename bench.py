@@ -202,7 +202,7 @@ def main() -> None:
     real64 = "double"
     dom = max(st64, key=lambda k: st64[k])
     roof = roofline_of(dom, st64, 16, "fp64")
-    roof["kernel_name"] = stage_kernel(dom, real64, wl.name)
+    roof["kernel_name"] = stage_kernel(dom, real64, wl.shape, info["fused_planes"])
     roof["traffic"], roof["traffic_source"] = profiled_traffic(args.workload, dom, real64)
     roof["stage_ms_fp64"] = st64
     roof["stage_ms_fp32"] = st32
@@ -803,8 +803,12 @@ def forces_check(wl, psi64, psims, psisw=None) -> dict:
             "band_energy_fixed_psi_eV": float(e64)}
 
 
-STAGE_KERNEL = {"plane_inv": "k_plane_inv_w", "xpass": "k_xpass_wave", "plane_fwd": "k_plane_fwd_w",
-                "becp": "k_gemm_inner_lds", "dmul": "k_dmul", "backproj": "k_gemm_combine_lds"}
+# kernels of the local-term stages: cubes of 90 and 120, other wave-line boxes, boxes
+# whose x-planes fit LDS, the rest (by gw_plan_info fused_planes)
+BOX_KERNELS = {"cube": ("k_plane_inv_w", "k_xpass_wave", "k_plane_fwd_w"),
+               2: ("k_plane_inv_any", "k_xpass_wave", "k_plane_fwd_any"),
+               1: ("k_plane_inv", "k_xpass", "k_plane_fwd"),
+               0: ("k_plane_inv_y", "k_xpass", "k_plane_fwd_y")}
 PROFILE_OF = {"si64_gamma": "hpsi_apply_si64_gamma_90cubed.txt",
               "si216_gamma": "hpsi_apply_si216_gamma_120cubed.txt"}
 
@@ -817,7 +821,8 @@ CTILE = {6: ((2, 2), (2, 2), False), 7: ((3, 3), (3, 2), False), 8: ((2, 5), (5,
 
 def gemm_mfma_fraction(stage: str, real: str) -> float:
     """Real MFMA flops per 8 algorithmic flops of the projector contraction that
-    runs ``stage``: 0.75 for the three-product tiles, 1 otherwise."""
+    runs ``stage``: 0.75 for the three-product tiles (explicit variants only; the
+    rule by shape has four products), 1 otherwise."""
     from gradwave_amd import _lib as L
 
     prec = L.GW_FP32 if real == "float" else L.GW_FP64
@@ -828,27 +833,37 @@ def gemm_mfma_fraction(stage: str, real: str) -> float:
     return 0.75 if tile in CTILE and CTILE[tile][2] else 1.0
 
 
-def stage_kernel(stage: str, real: str, workload: str = "") -> str:
-    """Kernel that runs a stage: the x pass is k_xpass_stage when the launch shape
-    of that precision stages the planes through LDS (mode digit of GW_TUNE_XPASS);
-    a projector contraction routed to rocBLAS by the autotuner runs its GEMM."""
+def stage_kernel(stage: str, real: str, shape, fused: int) -> str:
+    """Kernel that runs a stage on a box of this shape (``fused``: its
+    ``fused_planes``). The x pass of the 90 and 120 cubes is k_xpass_stage when the
+    launch shape of that precision stages the planes through LDS (mode digit of
+    GW_TUNE_XPASS), that of other wave-line boxes in FP32 where n2 n3 is even; a
+    projector contraction routed to rocBLAS by the autotuner runs its GEMM."""
     from gradwave_amd import _lib as L
 
     prec = L.GW_FP32 if real == "float" else L.GW_FP64
-    if stage == "xpass" and L.lib().gw_tune_get(L.GW_TUNE_XPASS, prec) // 10000 == 1:
+    cube = fused == 2 and len(set(shape)) == 1 and shape[0] in (90, 120)
+    box = dict(zip(("plane_inv", "xpass", "plane_fwd"), BOX_KERNELS["cube" if cube else fused]))
+    if stage == "xpass" and cube and L.lib().gw_tune_get(L.GW_TUNE_XPASS, prec) // 10000 == 1:
         return "k_xpass_stage"
-    if stage == "becp" and L.lib().gw_tune_get(L.GW_TUNE_INNER_LIB, prec):
+    if stage == "xpass" and fused == 2 and not cube and prec == L.GW_FP32 and shape[1] * shape[2] % 2 == 0:
+        return "k_xpass_stage (k_xpass_wave for few bands)"
+    if stage in box:
+        return box[stage]
+    if stage == "dmul":
+        return "k_dmul"
+    inner = stage == "becp"
+    if L.lib().gw_tune_get(L.GW_TUNE_INNER_LIB if inner else L.GW_TUNE_COMBINE_LIB, prec):
         return "rocBLAS " + ("zgemm" if prec == L.GW_FP64 else "cgemm") + " strided batched (Cijk_*)"
-    if stage == "backproj" and L.lib().gw_tune_get(L.GW_TUNE_COMBINE_LIB, prec):
-        return "rocBLAS " + ("zgemm" if prec == L.GW_FP64 else "cgemm") + " strided batched (Cijk_*)"
-    if stage in ("becp", "backproj"):
-        tile = L.lib().gw_tune_get(L.GW_TUNE_GEMM_TILE, prec + (256 if stage == "becp" else 512))
-        if tile in CTILE:
-            inner, comb, g3 = CTILE[tile]
-            bm, bn = inner if stage == "becp" else comb
-            return (f"k_cgemm_{'inner' if stage == 'becp' else 'combine'}<{real}, {bm}, {bn}, "
-                    f"{'true' if g3 else 'false'}{'' if stage == 'becp' else ', ...'}>")
-    return STAGE_KERNEL[stage]
+    op = "inner" if inner else "combine"
+    tile = L.lib().gw_tune_get(L.GW_TUNE_GEMM_TILE, prec + (256 if inner else 512))
+    if tile in CTILE:
+        ti, tc, g3 = CTILE[tile]
+        bm, bn = ti if inner else tc
+        return f"k_cgemm_{op}<{real}, {bm}, {bn}, {'true' if g3 else 'false'}{'' if inner else ', ...'}>"
+    if tile:
+        return f"k_gemm_{op}_tile<{real}, ...>"
+    return f"k_cgemm_{op}<{real}, ...> (tile by shape)"
 
 
 def profiled_traffic(workload: str, stage: str, real: str):
