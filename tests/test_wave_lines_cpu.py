@@ -1,4 +1,4 @@
-"""The wave-line x pass over every listed box length, on the host:
+"""The wave lines of every listed box length, on the host:
 tests/wave_lines_host.hip includes the headers of the kernels and is built here
 with hipcc."""
 
