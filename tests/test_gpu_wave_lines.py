@@ -42,3 +42,57 @@ def test_x_pass_of_large_blocks_matches_small_ones(n):
             assert torch.equal(got, _repeated(h.apply_terms(few, terms), nb))
             assert _rel(h.apply(many)[:, :_BANDS].cpu().to(torch.complex128), want) < tol
         _SYS.pop(shape)
+
+
+# y and z lines of every class of the plane kernels (largest part count 8, 10, 16)
+@pytest.mark.parametrize("shape", [(18, 24, 35), (20, 27, 64), (16, 90, 28), (21, 32, 100), (15, 75, 30), (18, 28, 160)])
+@pytest.mark.parametrize("dtype", [torch.complex128, torch.complex64])
+def test_planes_with_several_bands_per_item(shape, dtype):
+    """GW_TUNE_PLANE_BANDS 3 over 8 bands (the last item part-full) equals one band per
+    item to the bit, sphere padding included."""
+    s = _si2(shape)
+    cpu, _, h = _gpu_h(s, toeplitz="off")
+    assert h.info(dtype)["fused_planes"] == 2
+    say(f"plane bands {shape} {dtype}")
+    c = rand_block(cpu.nk, 8, cpu.npw_max, cpu.mask, seed=95).to(dev(), dtype)
+    terms, prec, lib = L.GW_TERM_KINETIC | L.GW_TERM_LOCAL, L.precision_of(dtype), L.lib()
+    try:
+        L.check(lib.gw_tune_set(L.GW_TUNE_PLANE_BANDS, prec, 1), "gw_tune_set")
+        one = h.apply_terms(c, terms)
+        L.check(lib.gw_tune_set(L.GW_TUNE_PLANE_BANDS, prec, 3), "gw_tune_set")
+        three = h.apply_terms(c, terms)
+    finally:
+        L.check(lib.gw_tune_set(L.GW_TUNE_PLANE_BANDS, prec, 0), "gw_tune_set")
+    assert torch.equal(three, one)
+    assert _rel(h.apply(c)[:, :3].cpu().to(torch.complex128), ref_h(s).apply(c[:, :3].cpu().to(torch.complex128))) < (
+        1e-12 if dtype == torch.complex128 else 2e-5)
+
+
+def _batch(shapes, flags=0):
+    from gradwave_amd.batching import RaggedBatch
+
+    hams, blocks, wants = [], [], []
+    for i, shape in enumerate(shapes):
+        s = _si2(shape)
+        cpu, _, h = _gpu_h(s, toeplitz="off", flags=flags)
+        c = rand_block(cpu.nk, 9 + i, cpu.npw_max, cpu.mask, seed=96 + i)
+        hams.append(h)
+        blocks.append(c)
+        wants.append(ref_h(s).apply(c))
+    return RaggedBatch(hams), hams, blocks, wants
+
+
+@pytest.mark.parametrize("shapes,fused", [
+    (((24, 30, 36), (112, 16, 27), (15, 75, 30), (20, 18, 160)), (2, 2, 2, 2)),  # parts up to 16
+    (((24, 30, 36), (14, 24, 30), (36, 36, 36)), (2, 1, 2)),                      # one cell without wave lines
+    (((14, 24, 30), (20, 25, 168)), (1, 1)),                                      # none with them
+])
+def test_ragged_batches_of_every_class(shapes, fused):
+    """The ragged wave-line passes of large part counts, and the generic passes that a
+    batch takes as a whole when a cell of it has no wave lines."""
+    batch, hams, blocks, wants = _batch(shapes)
+    for dtype, tol in ((torch.complex128, 1e-12), (torch.complex64, 2e-5)):
+        say(f"ragged batch {shapes} {dtype}")
+        assert tuple(h.info(dtype)["fused_planes"] for h in hams) == fused
+        for o, w in zip(batch.apply([c.to(dev(), dtype) for c in blocks]), wants):
+            assert _rel(o.cpu().to(torch.complex128), w) < tol
