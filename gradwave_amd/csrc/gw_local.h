@@ -142,6 +142,7 @@ inline bool wave_any_info(int n, int* lw, int* esize, int* smax) {
 
 int plane_bands_knob(bool fp32, bool inv);  // GW_TUNE_PLANE_BANDS, 0 unset
 template <typename T> bool wave_planes_fit(const Plan& P);
+template <typename T> int wave_planes_per_cu(const Plan& P);  // plane workgroups that a CU's LDS holds
 // the any-length wave lines take this plan's local term
 inline bool wave_any_ok(const Plan& P, int precision) {
   if ((P.flags & GW_PLAN_LEGACY) || !P.any_ok) return false;

@@ -475,6 +475,13 @@ template <typename T> bool wave_planes_fit(const Plan& P) {
   return any_plane_waves<T>(geom_of(&P, 1), (size_t)std::min(P.lds_max, kMaxLds), &emax) > 0;
 }
 
+template <typename T> int wave_planes_per_cu(const Plan& P) {
+  int emax;
+  const Geom g = geom_of(&P, 1);
+  const int nw = any_plane_waves<T>(g, (size_t)std::min(P.lds_max, kMaxLds), &emax);
+  return nw > 0 ? (int)(kLdsPerCu / any_plane_lds<T>(g, emax, nw)) : 0;
+}
+
 template <typename T> size_t wave_rag_plane_lds(const Geom& g, int* emax) {
   int lw, ey = 0, ez = 0, sm;
   if (!wave_any_info(g.n2, &lw, &ey, &sm) || !wave_any_info(g.n3, &lw, &ez, &sm)) return 0;
@@ -521,6 +528,7 @@ template <typename T> void wave_any_attrs(int want) {
                                   cpx<T>*, long, long, T, bool, hipStream_t);                                     \
   template void wave_any_attrs<T>(int);                                                                            \
   template bool wave_planes_fit<T>(const Plan&);                                                                   \
+  template int wave_planes_per_cu<T>(const Plan&);                                                                 \
   template size_t wave_rag_plane_lds<T>(const Geom&, int*);                                                        \
   template int wave_rag_planes<T>(bool, int, const RagInst<T>*, int, long, size_t, hipStream_t);
 

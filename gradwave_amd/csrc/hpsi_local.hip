@@ -1912,16 +1912,21 @@ static void set_generic_lds_attrs(int want) {
 
 // Bands per chunk of the local term when GW_TUNE_BAND_CHUNK leaves it open.
 // A box above the 256 MiB memory-side cache goes to HBM and back twice between the
-// passes; slices of at most 128 MiB stay in the cache. Only where that still leaves
-// each pass a few thousand workgroups of several a CU (stick rows up to 32 KiB): Si8,
-// 36 k-points, 24 bands of 36^3 FP64 (322 MB, 3 chunks) 424 -> 408 us. Boxes of 72^3
-// and up gain nothing: their passes then end in nearly empty last waves (Si64 90^3
-// FP32 in 3 chunks 772 -> 818 us, Si216 120^3 FP64 in 16 to 30 within 3% either way).
-static int auto_band_chunk(const Plan& P, int nb, size_t e) {
-  constexpr size_t kCache = size_t(256) << 20, kSlice = size_t(128) << 20, kRows = size_t(32) << 10;
+// passes; slices of at most 128 MiB stay in the cache, at the price of nearly empty last
+// waves of workgroups in each slice. That pays where a CU's LDS holds four plane
+// workgroups or more, whole / sliced us: 36^3 x 24 bands x 36 k FP64 445 / 429, 35^3 451 / 427, 30^3 x
+// 40 x 60 741 / 701, 45^3 x 24 x 36 1170 / 1140 (FP32 702 / 629), 72 x 35 x 35 x 40 x 20
+// FP32 579 / 513; from 1% less to 3% more at 32^3, 40^3, 48^3 and 50^3. With three or
+// fewer it does not: 60 x 60 x 30 x 70 x 7 954 / 970, 98 x 70 x 35 x 110 x 4 1825 / 1864 (FP32 1051 /
+// 1103), 70^3 x 400 FP32 1053 / 1084; the largest go both ways with the slice count
+// (105^3 x 470 FP32 7510 / 6800 in 16; 120^3 x 480 FP64 15005 / 14260 in 30, 17079 in 28).
+template <typename T>
+static int auto_band_chunk(const Plan& P, int nb) {
+  constexpr size_t kCache = size_t(256) << 20, kSlice = size_t(128) << 20;
   constexpr long kMinItems = 3072;
-  const size_t band = (size_t)P.nk * P.na * P.n[1] * P.n[2] * e;
-  if (band * nb <= kCache || (size_t)P.rows_max * (P.n[2] | 1) * e > kRows) return nb;
+  constexpr int kMinPerCu = 4;
+  const size_t band = (size_t)P.nk * P.na * P.n[1] * P.n[2] * sizeof(cpx<T>);
+  if (band * nb <= kCache || wave_planes_per_cu<T>(P) < kMinPerCu) return nb;
   const int chunks = (int)((band * nb + kSlice - 1) / kSlice);
   const int chunk = (nb + chunks - 1) / chunks;
   return (long)P.na * P.nk * chunk >= kMinItems ? chunk : nb;
@@ -1950,7 +1955,7 @@ static int apply_t(gw_plan* h, int terms, const cpx<T>* c, long ldc, long sc, cp
     if (int rc = require_box_fft(P, "the local term")) return rc;
     const int chunk0 = g_band_chunk[prec == GW_FP64 ? 0 : 1];
     const bool wave = !L.pencil_yc && wave_any_ok(P, prec) && !wave_path_ok(P, prec);
-    const int chunk = chunk0 > 0 ? std::min(chunk0, nb) : wave ? auto_band_chunk(P, nb, sizeof(cpx<T>)) : nb;
+    const int chunk = chunk0 > 0 ? std::min(chunk0, nb) : wave ? auto_band_chunk<T>(P, nb) : nb;
     for (int b0 = 0; b0 < nb; b0 += chunk) {  // band chunks (one pass sequence each)
       const int nbc = std::min(chunk, nb - b0);
       const Geom gc = geom_of(&P, nbc);
