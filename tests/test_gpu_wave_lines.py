@@ -96,3 +96,36 @@ def test_ragged_batches_of_every_class(shapes, fused):
         assert tuple(h.info(dtype)["fused_planes"] for h in hams) == fused
         for o, w in zip(batch.apply([c.to(dev(), dtype) for c in blocks]), wants):
             assert _rel(o.cpu().to(torch.complex128), w) < tol
+
+
+@pytest.mark.parametrize("shape", [(24, 24, 24), (36, 36, 36), (18, 24, 35), (20, 27, 64), (35, 70, 98), (21, 32, 100),
+                                   (72, 24, 72), (18, 28, 160)])
+@pytest.mark.parametrize("dtype", [torch.complex128, torch.complex64])
+def test_kinetic_term_is_rounded_once(shape, dtype):
+    """t c + V psi with V = 1 and t a thousand times as large: the result is within one
+    rounding of the exact sum, with a tenth of one for the local part (its transforms'
+    error, some ten roundings, a thousandth of the whole), so t c is not rounded by itself."""
+    import numpy as np
+
+    say(f"kinetic rounding {shape} {dtype}")
+    s = _si2(shape)
+    cpu, gpu, h = _gpu_h(s, toeplitz="off")
+    g = torch.Generator().manual_seed(97)
+    u = 2.0 ** (-53 if dtype == torch.complex128 else -24)
+    rdt = torch.float64 if dtype == torch.complex128 else torch.float32
+    t = (1000.0 * (1.0 + torch.rand(cpu.nk, cpu.npw_max, dtype=torch.float64, generator=g))).to(rdt).double()
+    h.plan.set_potential(torch.ones(shape, dtype=torch.float64, device=dev()))
+    h.plan.set_kinetic(t.to(dev()))
+    part = [(1.0 + torch.rand(cpu.nk, 9, cpu.npw_max, dtype=torch.float64, generator=g)).to(rdt) for _ in range(2)]
+    c = torch.complex(*part).to(dtype) * cpu.mask[:, None, :]
+    terms, prec, lib = L.GW_TERM_KINETIC | L.GW_TERM_LOCAL, L.precision_of(dtype), L.lib()
+    for bands in (1, 4):
+        try:
+            L.check(lib.gw_tune_set(L.GW_TUNE_PLANE_BANDS, prec, bands), "gw_tune_set")
+            got = h.apply_terms(c.to(dev()), terms).cpu()
+        finally:
+            L.check(lib.gw_tune_set(L.GW_TUNE_PLANE_BANDS, prec, 0), "gw_tune_set")
+        for have, x in ((got.real, c.real), (got.imag, c.imag)):
+            want = x.numpy().astype(np.longdouble) * (t[:, None, :].numpy().astype(np.longdouble) + 1)
+            err = np.abs(have.numpy().astype(np.longdouble) - want)
+            assert bool((err <= 1.1 * u * want).all()), float((err / np.maximum(u * want, 1e-300)).max())
