@@ -301,8 +301,8 @@ int gw_vloc_g_grad(int na, long npts, const double* positions, const int64_t* sp
  *   (`arg` ignored; 0 = default 2048).
  * GW_TUNE_GEMM_TILE: MFMA blocks per wave of the complex GEMMs; `arg` = precision
  *   (GW_FP64 / GW_FP32) + 256 * (0: both contractions, 1: inner only, 2: combine
- *   only; gw_tune_get with 0 reports the inner one); value 0 (default) = by shape, 1 = 4x2,
- *   2 = 2x4, 3 = 4x4; 4 and 5 cover 160
+ *   only; gw_tune_get with 0 reports the inner one); value 0 (default) = by shape,
+ *   four real products per complex one; 1 = 4x2, 2 = 2x4, 3 = 4x4; 4 and 5 cover 160
  *   bands (80 complex columns of the inner product, 160 rows of the
  *   back-projection) per workgroup: 4 = inner 2x5 / combine 5x2, 5 = inner 4x5 /
  *   combine 5x4. 6-13 are the complex-accumulator kernels (workgroup tile
@@ -327,9 +327,9 @@ int gw_vloc_g_grad(int na, long npts, const double* positions, const int64_t* sp
  *   band's transforms.
  * GW_TUNE_BAND_CHUNK: for precision `arg`, bands per chunk of the local term of
  *   gw_hpsi_apply (0, the default: the whole block, or slices of at most 128 MiB of
- *   a box above 256 MiB on the wave-line kernels); each chunk runs the three
- *   passes back to back on a box slice of that many bands; a value above 0 also sets the
- *   box part of gw_hpsi_workspace_bytes.
+ *   a box above 256 MiB on the wave-line kernels where four plane workgroups fit a
+ *   CU's LDS); each chunk runs the three passes back to back on a box slice of that
+ *   many bands; a value above 0 also sets the box part of gw_hpsi_workspace_bytes.
  * GW_TUNE_INNER_LIB: for precision `arg`, 1 runs the K-chunks of gw_zgemm_inner (and
  *   of the projection <beta|psi>) as one rocBLAS strided-batched GEMM whose partials the
  *   FP64 split-K reduction here sums, 0 the MFMA kernels here (default). */
